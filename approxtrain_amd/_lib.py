@@ -72,6 +72,8 @@ SIGNATURES = {
     "amsim_attention_grad_workspace_bytes": (_sz, [_i] * 5),
     "amsim_attention_grad_workspace_bytes_for": (_sz, [_p] + [_i] * 5),
     "amsim_attention_grad_f32": (_i, [_p, _f, _f, _f, _f, _f] + [_i] * 5 + [C.c_float, _f, _f, _f, _p, _sz, _p]),
+    "amsim_epilogue_grad_workspace_bytes": (_sz, [_i64, _i]),
+    "amsim_epilogue_grad_f32": (_i, [_f, _f, _i64, _i, _i, _f, _f, _p, _sz, _p]),
     "amsim_conv_geometry": (_i, [_i, _i, _i, _i, C.POINTER(_i), C.POINTER(_i)]),
     "amsim_set_split_k": (_i, [_i]),
     "amsim_set_engine": (_i, [_i]),

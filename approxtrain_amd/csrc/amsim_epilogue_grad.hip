@@ -1,0 +1,138 @@
+// Gradient of the fused epilogue act(z + bias) (amdenselayer.py:211-226, am_convolutional.py:248-276 run
+// BiasAdd and the activation as ops of their own): d(z) = d(out) masked by the rectifier, d(bias) = sum
+// of d(z) over the rows, in one pass over the gradient.
+//
+// HBM-bound: 4 bytes per element for a bias alone, 12 with the rectifier.  A workgroup owns a slab of
+// rows of up to 64 columns; its threads run along the columns first, so that a wavefront reads whole
+// 64-byte pieces even of the narrowest outputs in use, and each adds every (256 / columns)-th row in four
+// chains.  The slabs' sums go to the workspace and the fixed-order reduction adds them: no atomics, no
+// counter to clear, the same bits on every run.
+// Compare, product with the mask, fill and sum as separate passes took 23.0 us for LeNet-5's second layer
+// at batch 256 (25600 x 16), fill and sum 21.8 us for 8192 x 512.  With this file: that layer's training
+// step 193.4 -> 189.0 us, the 32 x 256 x 512 attention block's (four biases) 2707 -> 2652 us.
+#include "amsim_internal.h"
+#include "amsim_device.h"
+#include "amsim_gemm_common.h"
+
+#include <algorithm>
+
+namespace amsim {
+
+namespace {
+
+constexpr int WG = 256;
+constexpr int ROWS_PER_THREAD = 16;  // shortest slab: four loads in flight, four times
+constexpr int MAX_SLABS = 2048;      // then slabs grow instead: eight workgroups per compute unit
+
+struct EpilogueGradArgs {
+    const float *grad, *out;  // out: only with the rectifier
+    float *grad_z, *partial;  // [rows][cols]; [slabs][cols] or null
+    int64_t rows, rows_per_slab;
+    int cols;
+};
+
+inline int threads_along_columns(int cols) { return cols > 32 ? 64 : cols > 16 ? 32 : 16; }
+
+inline int64_t slabs_of(int64_t rows, int cols)
+{
+    const int64_t shortest = (int64_t)(WG / threads_along_columns(cols)) * ROWS_PER_THREAD;
+    return std::min<int64_t>((rows + shortest - 1) / shortest, MAX_SLABS);
+}
+
+template <int TX, bool RELU>
+__global__ __launch_bounds__(WG) void epilogue_grad_kernel(EpilogueGradArgs a)
+{
+    constexpr int TY = WG / TX;
+    __shared__ float part[TY][TX];
+    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+    const int64_t col = (int64_t)blockIdx.x * TX + tx;
+    const int64_t beg = (int64_t)blockIdx.y * a.rows_per_slab;
+    const int64_t end = beg + a.rows_per_slab < a.rows ? beg + a.rows_per_slab : a.rows;
+    float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (col < a.cols) {
+        for (int64_t r = beg + ty; r < end; r += 4 * TY) {
+            float g[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t i = (r + u * TY) * a.cols + col;
+                g[u] = r + u * TY < end ? a.grad[i] : 0.0f;
+                // (a product with the mask, not a select: an infinite gradient of a masked element gives NaN)
+                if (RELU && r + u * TY < end) g[u] = g[u] * (a.out[i] > 0.0f ? 1.0f : 0.0f);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (RELU && r + u * TY < end) a.grad_z[(r + u * TY) * a.cols + col] = g[u];
+                c[u] += g[u];
+            }
+        }
+    }
+    if (a.partial == nullptr) return;  // (the same for every thread)
+    part[ty][tx] = (c[0] + c[1]) + (c[2] + c[3]);
+    __syncthreads();
+    if (ty == 0 && col < a.cols) {
+        float s = part[0][tx];
+#pragma unroll
+        for (int w = 1; w < TY; ++w) s += part[w][tx];
+        a.partial[(int64_t)blockIdx.y * a.cols + col] = s;
+    }
+}
+
+template <int TX>
+void launch_epilogue_grad(const EpilogueGradArgs &a, int64_t slabs, bool relu, hipStream_t stream)
+{
+    const dim3 grid((unsigned)((a.cols + TX - 1) / TX), (unsigned)slabs);
+    if (relu) epilogue_grad_kernel<TX, true><<<grid, WG, 0, stream>>>(a);
+    else epilogue_grad_kernel<TX, false><<<grid, WG, 0, stream>>>(a);
+}
+
+}  // namespace
+
+}  // namespace amsim
+
+using namespace amsim;
+
+extern "C" {
+
+size_t amsim_epilogue_grad_workspace_bytes(int64_t rows, int cols)
+{
+    if (rows <= 0 || cols <= 0) return 0;
+    return (size_t)slabs_of(rows, cols) * (size_t)cols * sizeof(float);
+}
+
+int amsim_epilogue_grad_f32(const float *grad, const float *out, int64_t rows, int cols, int act, float *grad_z,
+                            float *grad_bias, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (rows < 0 || cols < 0) return fail(AMSIM_ERR_INVALID, "negative extent");
+    if (act != AMSIM_ACT_NONE && act != AMSIM_ACT_RELU) return fail(AMSIM_ERR_INVALID, "unknown activation");
+    const bool relu = act == AMSIM_ACT_RELU;
+    if (rows == 0 || cols == 0) return fail(AMSIM_ERR_INVALID, "empty gradient");
+    if (!relu && !grad_bias) return AMSIM_OK;
+    if (!grad || (relu && (!out || !grad_z))) return fail(AMSIM_ERR_INVALID, "null tensor pointer");
+    const size_t need = grad_bias ? amsim_epilogue_grad_workspace_bytes(rows, cols) : 0;
+    if (need && (workspace == nullptr || ((uintptr_t)workspace & 255) || workspace_bytes < need))
+        return fail(AMSIM_ERR_WORKSPACE, "workspace missing, not 256-byte aligned or smaller than " +
+                                             std::to_string(need) + " bytes");
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t slabs = slabs_of(rows, cols);
+    EpilogueGradArgs a{grad, out, grad_z, grad_bias ? static_cast<float *>(workspace) : nullptr, rows,
+                       (rows + slabs - 1) / slabs, cols};
+    switch (threads_along_columns(cols)) {
+    case 64: launch_epilogue_grad<64>(a, slabs, relu, s); break;
+    case 32: launch_epilogue_grad<32>(a, slabs, relu, s); break;
+    default: launch_epilogue_grad<16>(a, slabs, relu, s); break;
+    }
+    AMSIM_HIP_CHECK(hipGetLastError());
+    if (!grad_bias) return AMSIM_OK;
+    RArgs ra{};
+    ra.partial = a.partial;
+    ra.out = grad_bias;
+    ra.R = 1; ra.J = cols; ra.Rp = 1; ra.Jp = cols;
+    ra.so_r = cols; ra.so_j = 1;
+    ra.nsplit = (int)slabs;
+    ra.batch = 1;
+    launch_reduce(ra, s);
+    AMSIM_HIP_CHECK(hipGetLastError());
+    return AMSIM_OK;
+}
+
+}  // extern "C"

@@ -310,3 +310,21 @@ def attention_grad(lut, q, k, v, weights, grad_out, divisor):
                                        sq, sk, dk, dv, float(divisor), _ptr(gq), _ptr(gk), _ptr(gv), wsp, nbytes,
                                        _stream()))
     return gq, gk, gv
+
+
+def epilogue_grad(grad, out, has_bias, activation):
+    """Gradient of ``activation(z + bias)`` given its output: (dL/dz, dL/dbias or None)."""
+    grad = _dev(grad, "grad")
+    relu = activation == "relu"
+    cols = grad.shape[-1]
+    rows = grad.numel() // cols
+    out = _dev(out, "out") if relu else None
+    grad_z = torch.empty_like(grad) if relu else grad
+    grad_bias = torch.empty(cols, dtype=torch.float32, device=grad.device) if has_bias else None
+    lib = load_library()
+    nbytes = lib.amsim_epilogue_grad_workspace_bytes(rows, cols) if has_bias else 0
+    ws, wsp = _workspace(nbytes, grad.device)
+    check(lib.amsim_epilogue_grad_f32(_ptr(grad), _ptr(out) if relu else None, rows, cols, int(relu),
+                                      _ptr(grad_z) if relu else None, _ptr(grad_bias) if has_bias else None, wsp,
+                                      nbytes, _stream()))
+    return grad_z, grad_bias

@@ -139,6 +139,11 @@ class _KerasLayerArgs:
 def _epilogue_backward(grad, out, bias, act):
     """Gradient through act(z + bias) given its output: (dL/dz, dL/dbias)."""
     grad = grad.contiguous()
+    # (a gradient that is itself recorded for differentiation, empty or not in 32 bits takes torch's ops)
+    if grad.is_cuda and grad.dtype == torch.float32 and grad.numel() and not torch.is_grad_enabled():
+        if bias is None and act != "relu":
+            return grad, None
+        return functors.epilogue_grad(grad, out, bias is not None, act)
     if act == "relu":
         grad = grad * (out > 0)
     grad_bias = grad.reshape(-1, grad.shape[-1]).sum(0) if bias is not None else None

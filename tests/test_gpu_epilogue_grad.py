@@ -1,0 +1,35 @@
+"""Gradient of the fused bias + ReLU epilogue: edges of the column tiles, of the rows per slab and of the slab count."""
+import pytest
+import torch
+
+from approxtrain_amd import functors
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 16), (255, 17), (256, 6), (257, 16), (129, 33), (64, 64), (65, 65),
+                                       (1000, 513), (25600, 16), (140000, 70), (600001, 3)])
+@pytest.mark.parametrize("act", ["relu", None])
+@pytest.mark.parametrize("has_bias", [True, False])
+def test_epilogue_grad(rows, cols, act, has_bias):
+    gen = torch.Generator().manual_seed(rows * 1000 + cols)
+    grad, out = torch.randn(rows, cols, generator=gen), torch.randn(rows, cols, generator=gen).relu_()
+    z, b = functors.epilogue_grad(grad.cuda(), out.cuda(), has_bias, act)
+    want = grad * (out > 0) if act == "relu" else grad
+    assert torch.equal(z.cpu(), want)
+    assert (b is None) == (not has_bias)
+    if has_bias:
+        # every 32-bit sum of n terms lies within n * 2^-24 * sum|terms|; slabs, chains and ways cut the n of
+        # any one chain below 1024 (rows of a slab per chain + ways + slabs per chain)
+        bound = 1024 * 2.0 ** -24 * want.double().abs().sum(0)
+        assert ((b.cpu().double() - want.double().sum(0)).abs() <= bound).all()
+        again = functors.epilogue_grad(grad.cuda(), out.cuda(), True, act)[1]
+        assert torch.equal(b, again)
+
+
+def test_infinite_gradient_of_a_masked_element_is_nan():
+    grad = torch.tensor([[float("inf"), 1.0], [2.0, float("nan")]]).cuda()
+    out = torch.tensor([[0.0, 1.0], [1.0, float("nan")]]).cuda()
+    z, b = functors.epilogue_grad(grad, out, True, "relu")
+    assert torch.equal(torch.isnan(z).cpu(), torch.tensor([[True, False], [False, True]]))
+    assert torch.isnan(b).all()
