@@ -314,8 +314,11 @@ def attention_grad(lut, q, k, v, weights, grad_out, divisor):
 
 def epilogue_grad(grad, out, has_bias, activation):
     """Gradient of ``activation(z + bias)`` given its output: (dL/dz, dL/dbias or None)."""
+    if activation not in ACTIVATIONS:
+        raise ValueError("fused activation must be None, 'linear' or 'relu'")
+    act = ACTIVATIONS[activation]
     grad = _dev(grad, "grad")
-    relu = activation == "relu"
+    relu = act == ACTIVATIONS["relu"]
     cols = grad.shape[-1]
     rows = grad.numel() // cols
     out = _dev(out, "out") if relu else None
@@ -324,7 +327,7 @@ def epilogue_grad(grad, out, has_bias, activation):
     lib = load_library()
     nbytes = lib.amsim_epilogue_grad_workspace_bytes(rows, cols) if has_bias else 0
     ws, wsp = _workspace(nbytes, grad.device)
-    check(lib.amsim_epilogue_grad_f32(_ptr(grad), _ptr(out) if relu else None, rows, cols, int(relu),
+    check(lib.amsim_epilogue_grad_f32(_ptr(grad), _ptr(out) if relu else None, rows, cols, act,
                                       _ptr(grad_z) if relu else None, _ptr(grad_bias) if has_bias else None, wsp,
                                       nbytes, _stream()))
     return grad_z, grad_bias
