@@ -317,11 +317,16 @@ def epilogue_grad(grad, out, has_bias, activation):
     if activation not in ACTIVATIONS:
         raise ValueError("fused activation must be None, 'linear' or 'relu'")
     act = ACTIVATIONS[activation]
-    grad = _dev(grad, "grad")
     relu = act == ACTIVATIONS["relu"]
+    # the kernel reads and writes whole tensors of the gradient's extents
+    if relu and out.shape != grad.shape:
+        raise ValueError("out must have the gradient's shape")
+    grad = _dev(grad, "grad")
     cols = grad.shape[-1]
     rows = grad.numel() // cols
     out = _dev(out, "out") if relu else None
+    if relu and out.device != grad.device:
+        raise ValueError("out must be on the gradient's device")
     grad_z = torch.empty_like(grad) if relu else grad
     grad_bias = torch.empty(cols, dtype=torch.float32, device=grad.device) if has_bias else None
     lib = load_library()
