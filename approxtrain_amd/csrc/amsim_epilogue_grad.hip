@@ -26,7 +26,7 @@ constexpr int MAX_SLABS = 2048;      // then slabs grow instead: eight workgroup
 
 struct EpilogueGradArgs {
     const float *grad, *out;  // out: only with the rectifier
-    float *grad_z, *partial;  // [rows][cols]; [slabs][cols] or null
+    float *grad_z, *partial;  // [rows][cols]; [slabs][cols] (one slab: d(bias) itself) or null
     int64_t rows, rows_per_slab;
     int cols;
 };
@@ -96,7 +96,8 @@ extern "C" {
 size_t amsim_epilogue_grad_workspace_bytes(int64_t rows, int cols)
 {
     if (rows <= 0 || cols <= 0) return 0;
-    return (size_t)slabs_of(rows, cols) * (size_t)cols * sizeof(float);
+    const int64_t slabs = slabs_of(rows, cols);
+    return slabs == 1 ? 0 : (size_t)slabs * (size_t)cols * sizeof(float);
 }
 
 int amsim_epilogue_grad_f32(const float *grad, const float *out, int64_t rows, int cols, int act, float *grad_z,
@@ -114,15 +115,16 @@ int amsim_epilogue_grad_f32(const float *grad, const float *out, int64_t rows, i
                                              std::to_string(need) + " bytes");
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t slabs = slabs_of(rows, cols);
-    EpilogueGradArgs a{grad, out, grad_z, grad_bias ? static_cast<float *>(workspace) : nullptr, rows,
-                       (rows + slabs - 1) / slabs, cols};
+    // one slab's sums are the bias gradient: no workspace and no second launch, which would only copy them
+    float *const partial = !grad_bias ? nullptr : slabs == 1 ? grad_bias : static_cast<float *>(workspace);
+    EpilogueGradArgs a{grad, out, grad_z, partial, rows, (rows + slabs - 1) / slabs, cols};
     switch (threads_along_columns(cols)) {
     case 64: launch_epilogue_grad<64>(a, slabs, relu, s); break;
     case 32: launch_epilogue_grad<32>(a, slabs, relu, s); break;
     default: launch_epilogue_grad<16>(a, slabs, relu, s); break;
     }
     AMSIM_HIP_CHECK(hipGetLastError());
-    if (!grad_bias) return AMSIM_OK;
+    if (!grad_bias || slabs == 1) return AMSIM_OK;
     RArgs ra{};
     ra.partial = a.partial;
     ra.out = grad_bias;

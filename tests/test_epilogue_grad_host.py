@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from approxtrain_amd import functors
+from approxtrain_amd import functors, load_library
 
 
 @pytest.mark.parametrize("activation", ["sigmoid", "Relu", 1])
@@ -16,3 +16,11 @@ def test_unknown_activation_is_refused(activation):
 def test_output_of_another_shape_is_refused(shape):
     with pytest.raises(ValueError, match="shape"):
         functors.epilogue_grad(torch.zeros(2, 3), torch.zeros(shape), True, "relu")
+
+
+@pytest.mark.parametrize("cols,shortest", [(1, 256), (16, 256), (17, 128), (32, 128), (33, 64), (4096, 64)])
+def test_one_slab_needs_no_workspace(cols, shortest):
+    """Rows that one workgroup adds go to the bias gradient at once: nothing to reduce, nothing to allocate."""
+    query = load_library().amsim_epilogue_grad_workspace_bytes
+    assert query(1, cols) == 0 and query(shortest, cols) == 0
+    assert query(shortest + 1, cols) == 2 * cols * 4
