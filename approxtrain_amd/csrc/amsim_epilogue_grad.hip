@@ -31,6 +31,10 @@ struct EpilogueGradArgs {
     int cols;
 };
 
+// The grid's first extent times the workgroup's threads stays below 2^32 (here and in the reduction of the
+// slabs, four threads per column each), element indices far below 2^63.
+inline bool extents_fit(int64_t rows, int cols) { return cols < (1 << 30) && (double)rows * cols <= 17592186044416.0; }
+
 inline int threads_along_columns(int cols) { return cols > 32 ? 64 : cols > 16 ? 32 : 16; }
 
 inline int64_t slabs_of(int64_t rows, int cols)
@@ -95,7 +99,7 @@ extern "C" {
 
 size_t amsim_epilogue_grad_workspace_bytes(int64_t rows, int cols)
 {
-    if (rows <= 0 || cols <= 0) return 0;
+    if (rows <= 0 || cols <= 0 || !extents_fit(rows, cols)) return 0;
     const int64_t slabs = slabs_of(rows, cols);
     return slabs == 1 ? 0 : (size_t)slabs * (size_t)cols * sizeof(float);
 }
@@ -105,6 +109,7 @@ int amsim_epilogue_grad_f32(const float *grad, const float *out, int64_t rows, i
 {
     if (rows < 0 || cols < 0) return fail(AMSIM_ERR_INVALID, "negative extent");
     if (act != AMSIM_ACT_NONE && act != AMSIM_ACT_RELU) return fail(AMSIM_ERR_INVALID, "unknown activation");
+    if (!extents_fit(rows, cols)) return fail(AMSIM_ERR_UNSUPPORTED, "gradient exceeds the grid limit");
     const bool relu = act == AMSIM_ACT_RELU;
     if (rows == 0 || cols == 0) return fail(AMSIM_ERR_INVALID, "empty gradient");
     if (!relu && !grad_bias) return AMSIM_OK;

@@ -24,3 +24,12 @@ def test_one_slab_needs_no_workspace(cols, shortest):
     query = load_library().amsim_epilogue_grad_workspace_bytes
     assert query(1, cols) == 0 and query(shortest, cols) == 0
     assert query(shortest + 1, cols) == 2 * cols * 4
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1 << 30), (1 << 44, 3), (1 << 62, 4)])
+def test_extents_beyond_the_grid_are_refused(rows, cols):
+    lib = load_library()
+    assert lib.amsim_epilogue_grad_workspace_bytes(rows, cols) == 0
+    # (act NONE without a bias gradient: an accepted call has nothing to launch)
+    assert lib.amsim_epilogue_grad_f32(None, None, rows, cols, 0, None, None, None, 0, None) == 6
+    assert lib.amsim_epilogue_grad_f32(None, None, 1 << 20, 1 << 20, 0, None, None, None, 0, None) == 0
