@@ -322,12 +322,16 @@ def epilogue_grad(grad, out, has_bias, activation):
     if relu and isinstance(out, torch.Tensor) and out.shape != grad.shape:
         raise ValueError("out must have the gradient's shape")
     grad = _dev(grad, "grad")
+    if grad.dim() == 0:
+        raise ValueError("grad needs a last dimension, the bias's")
     cols = grad.shape[-1]
-    rows = grad.numel() // cols
     out = _dev(out, "out") if relu else None
     if relu and out.device != grad.device:
         raise ValueError("out must be on the gradient's device")
     grad_z = torch.empty_like(grad) if relu else grad
+    if grad.numel() == 0:
+        return grad_z, torch.zeros(cols, dtype=torch.float32, device=grad.device) if has_bias else None
+    rows = grad.numel() // cols
     grad_bias = torch.empty(cols, dtype=torch.float32, device=grad.device) if has_bias else None
     lib = load_library()
     nbytes = lib.amsim_epilogue_grad_workspace_bytes(rows, cols) if has_bias else 0

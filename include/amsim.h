@@ -292,7 +292,7 @@ int amsim_attention_grad_f32(amsim_lut_t lut, const float *q, const float *k, co
  * grad: d(out) as [rows][cols], cols the bias's length.  act = RELU: grad_z = grad * (out > 0); act =
  * NONE: out and grad_z are not touched and d(z) is grad itself.  grad_bias (optional) receives the sum of
  * d(z) over the rows, in a fixed order.  The workspace (with grad_bias, where the query says so: few rows
- * need none) is 256-byte aligned. */
+ * need none) is 256-byte aligned.  Refused (AMSIM_ERR_INVALID): rows or cols of 0, nothing to run on. */
 size_t amsim_epilogue_grad_workspace_bytes(int64_t rows, int cols);
 int amsim_epilogue_grad_f32(const float *grad, const float *out, int64_t rows, int cols, int act, float *grad_z,
                             float *grad_bias, void *workspace, size_t workspace_bytes, void *stream);

@@ -33,3 +33,10 @@ def test_extents_beyond_the_grid_are_refused(rows, cols):
     # (act NONE without a bias gradient: an accepted call has nothing to launch)
     assert lib.amsim_epilogue_grad_f32(None, None, rows, cols, 0, None, None, None, 0, None) == 6
     assert lib.amsim_epilogue_grad_f32(None, None, 1 << 20, 1 << 20, 0, None, None, None, 0, None) == 0
+
+
+@pytest.mark.parametrize("rows,cols", [(0, 3), (3, 0), (0, 0)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_empty_gradients_are_refused_at_the_boundary(rows, cols, act):
+    """As the header says (functors.epilogue_grad answers them itself)."""
+    assert load_library().amsim_epilogue_grad_f32(None, None, rows, cols, act, None, None, None, 0, None) == 1

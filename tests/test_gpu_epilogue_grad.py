@@ -33,3 +33,11 @@ def test_infinite_gradient_of_a_masked_element_is_nan():
     z, b = functors.epilogue_grad(grad, out, True, "relu")
     assert torch.equal(torch.isnan(z).cpu(), torch.tensor([[True, False], [False, True]]))
     assert torch.isnan(b).all()
+
+
+@pytest.mark.parametrize("shape", [(0, 3), (2, 0, 70), (3, 0), (0,)])
+@pytest.mark.parametrize("act", ["relu", None])
+def test_empty_gradient(shape, act):
+    grad = torch.empty(shape).cuda()
+    z, b = functors.epilogue_grad(grad, torch.empty(shape).cuda(), True, act)
+    assert z.shape == grad.shape and torch.equal(b.cpu(), torch.zeros(shape[-1]))
