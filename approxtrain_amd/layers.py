@@ -9,6 +9,7 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 
 from . import functors
 from .amnn_ops import amconvolution_v2
@@ -136,13 +137,36 @@ class _KerasLayerArgs:
                 self.bias.copy_(self.bias_constraint(self.bias))
 
 
+def _plain_memory(t):
+    """Whether the values of ``t`` are 32-bit floats that lie in device memory as they are: not a
+    subclass's, a batched (vmap), lazily negated or lazily zero tensor's."""
+    if type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.float32 or t.is_neg():
+        return False
+    try:
+        return t.data_ptr() != 0
+    except RuntimeError:
+        return False
+
+
+def _library_epilogue(grad, out):
+    """Whether the epilogue's gradient may go to the library, which reads memory where torch's
+    operations would see everything else that is going on: a backward pass that is itself recorded
+    (for differentiation or by a dispatch mode), a forward-mode tangent, or a saved output (``out``,
+    None where it is not read) that a hook brought back in another form.  Empty gradients and such
+    wider than the library's grid are torch's as well."""
+    if torch.is_grad_enabled() or torch._C._len_torch_dispatch_stack() or not grad.numel():
+        return False
+    if not _plain_memory(grad) or grad.shape[-1] >= 1 << 30 or forward_ad.unpack_dual(grad).tangent is not None:
+        return False
+    return out is None or (_plain_memory(out) and out.shape == grad.shape and out.device == grad.device)
+
+
 def _epilogue_backward(grad, out, bias, act):
     """Gradient through act(z + bias) given its output: (dL/dz, dL/dbias)."""
     grad = grad.contiguous()
-    # (a gradient that is itself recorded for differentiation, empty or not in 32 bits takes torch's ops)
-    if grad.is_cuda and grad.dtype == torch.float32 and grad.numel() and not torch.is_grad_enabled():
-        if bias is None and act != "relu":
-            return grad, None
+    if bias is None and act != "relu":
+        return grad, None
+    if _library_epilogue(grad, out if act == "relu" else None):
         return functors.epilogue_grad(grad, out, bias is not None, act)
     if act == "relu":
         grad = grad * (out > 0)
