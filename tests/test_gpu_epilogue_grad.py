@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from approxtrain_amd import functors
+from approxtrain_amd import functors, layers
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +41,19 @@ def test_empty_gradient(shape, act):
     grad = torch.empty(shape).cuda()
     z, b = functors.epilogue_grad(grad, torch.empty(shape).cuda(), True, act)
     assert z.shape == grad.shape and torch.equal(b.cpu(), torch.zeros(shape[-1]))
+
+
+@pytest.mark.parametrize("rows,cols,act,calls", [(1, 1, None, 0), (80, 128, None, 0), (4095, 512, None, 0),
+                                                 (4096, 512, None, 1), (80, 128, "relu", 1), (4096, 512, "relu", 1)])
+def test_small_gradients_of_a_bias_alone_stay_with_torch(monkeypatch, rows, cols, act, calls):
+    seen = []
+    library = functors.epilogue_grad_checked
+    monkeypatch.setattr(functors, "epilogue_grad_checked", lambda *a: seen.append(a) or library(*a))
+    gen = torch.Generator(device="cuda").manual_seed(rows + cols)
+    grad, out = (torch.randn((rows, cols), device="cuda", generator=gen) for _ in range(2))
+    with torch.no_grad():
+        z, b = layers._epilogue_backward(grad, out, True, act)
+    want = grad * (out > 0) if act == "relu" else grad
+    assert torch.equal(z, want) and len(seen) == calls
+    # (any order of the sum: n * 2^-24 * sum|terms|)
+    assert ((b.double() - want.double().sum(0)).abs() <= rows * 2.0 ** -24 * want.double().abs().sum(0)).all()
