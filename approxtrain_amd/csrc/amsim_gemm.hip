@@ -1002,14 +1002,21 @@ void launch_reduce(const RArgs &ra, hipStream_t stream)
         return;
     }
     // up to four slices: every way of the general kernel holds at most one, added in slice order -- the
-    // same sum, bit for bit.  Below 2^16 outputs both are a launch's length.
+    // same sum, bit for bit.  A thread per output is ahead of the general kernel from 4096 outputs on
+    // (2.2 us against 2.4; 65536: 2.3 / 2.7; 2049 x 515: 4.4 / 11.7), and the line stands at 2^16 because below it
+    // both are a launch's length.
     if (ra.nsplit <= SHALLOW_SLICES && outs * ra.batch >= (1 << 16) && outs < (1ll << 31)) {
+        // Outputs along the rows turn where that pays (three slices, thread per output / turned / general): 4096 x 128
+        // 7.9 / 4.6 / 8.6 us, 8200 x 64 5.7 / 4.7 / 9.3, 64 x 8192 4.7 / 4.5 / 7.2.  Not with fewer outputs (256 x 256: 2.9 / 4.1 /
+        // 2.9; 512 x 513: 4.1 / 4.4 / 4.8), few columns, whose stores the L2 merges (16 x 4097 x 17: 7.2 / 11.7 / 14.3), or tiles
+        // mostly empty (16 x 3 x 21846: 6.1 / 31.6 / 12.9; 65 x 8192: 4.7 / 5.4 / 7.2).
         const int64_t turn_tiles = ((ra.R + TURN_ROWS - 1) / TURN_ROWS) * ((ra.J + TURN_COLS - 1) / TURN_COLS);
-        if (ra.so_r == 1 && ra.so_j != 1 && !ra.ep.omap.enabled) {
+        const bool turn = ra.so_r == 1 && ra.so_j != 1 && !ra.ep.omap.enabled && outs * ra.batch >= (1 << 19) &&
+                          ra.J >= 4 * TURN_COLS && 3 * outs >= 2 * turn_tiles * TURN_ROWS * TURN_COLS;
+        if (turn)
             splitk_reduce_turn_kernel<<<dim3((unsigned)turn_tiles, (unsigned)ra.batch), WG_THREADS, 0, stream>>>(ra);
-            return;
-        }
-        splitk_reduce_shallow_kernel<<<dim3((unsigned)((outs + WG_THREADS - 1) / WG_THREADS), (unsigned)ra.batch), WG_THREADS, 0, stream>>>(ra);
+        else
+            splitk_reduce_shallow_kernel<<<dim3((unsigned)((outs + WG_THREADS - 1) / WG_THREADS), (unsigned)ra.batch), WG_THREADS, 0, stream>>>(ra);
         return;
     }
     if (outs * ra.batch <= 16384 && ra.nsplit >= 64)
