@@ -3,13 +3,15 @@
 // of d(z) over the rows, in one pass over the gradient.
 //
 // HBM-bound: 4 bytes per element for a bias alone, 12 with the rectifier.  A workgroup owns a slab of
-// rows of up to 64 columns; its threads run along the columns first, so that a wavefront reads whole
-// 64-byte pieces even of the narrowest outputs in use, and each adds every (256 / columns)-th row in four
-// chains.  The slabs' sums go to the workspace and the fixed-order reduction adds them: no atomics, no
-// counter to clear, the same bits on every run.
-// Compare, product with the mask, fill and sum as separate passes took 23.0 us for LeNet-5's second layer
-// at batch 256 (25600 x 16), fill and sum 21.8 us for 8192 x 512.  With this file: that layer's training
-// step 193.4 -> 189.0 us, the 32 x 256 x 512 attention block's (four biases) 2707 -> 2652 us.
+// rows of up to 64 columns; its threads run along the columns first, 16 lanes or more, and each adds every
+// (256 / columns)-th row in four chains.  Rows of fewer than 16 columns leave lanes idle (6 columns: ten of
+// 16) and are read in short pieces, which a narrow output's few bytes bear.  The slabs' sums go to the workspace and
+// the fixed-order reduction adds them (one slab writes the bias gradient itself): no atomics, no counter to
+// clear, the same bits on every run.
+// On the device, torch's compare, product with the mask and sum against this file: 25600 x 16 18.4 -> 8.4 us,
+// 401408 x 6 30.6 -> 13.6, 8192 x 512 37.7 -> 14.7 (3.4 TB/s), 401408 x 128 257 -> 129 (4.8 TB/s); the sum alone
+// 8192 x 512 17.8 -> 8.1, 401408 x 128 52.4 -> 37.3 (5.5 TB/s).  Training step of the 32 x 256 x 512 attention block
+// (four biases) 2711 -> 2661 us; LeNet-5's convolutions, bound by the host, show no difference beyond their spread.
 #include "amsim_internal.h"
 #include "amsim_device.h"
 #include "amsim_gemm_common.h"
@@ -22,7 +24,7 @@ namespace {
 
 constexpr int WG = 256;
 constexpr int ROWS_PER_THREAD = 16;  // shortest slab: four loads in flight, four times
-constexpr int MAX_SLABS = 2048;      // then slabs grow instead: eight workgroups per compute unit
+constexpr int MAX_SLABS = 2048;      // then slabs grow instead: eight workgroups per compute unit and column tile
 
 struct EpilogueGradArgs {
     const float *grad, *out;  // out: only with the rectifier
