@@ -347,5 +347,5 @@ def epilogue_grad_checked(grad, out, has_bias, act):
     check(lib.amsim_epilogue_grad_f32(grad.data_ptr(), out.data_ptr() if act else None, rows, cols, act,
                                       grad_z.data_ptr() if act else None, grad_bias.data_ptr() if has_bias else None,
                                       ws.data_ptr() if nbytes else None, nbytes,
-                                      torch._C._cuda_getCurrentRawStream(grad.get_device())))
+                                      torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())))
     return grad_z, grad_bias
