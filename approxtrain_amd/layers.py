@@ -162,8 +162,13 @@ def _library_epilogue(grad, out):
     operations would see everything else that is going on: a backward pass that is itself recorded
     (for differentiation or by a dispatch mode), a forward-mode tangent, or a saved output (``out``,
     None where it is not read) that a hook brought back in another form.  Empty gradients and such
-    wider than the library's grid are torch's as well, and few elements without a rectifier."""
-    if grad.numel() < (_BIAS_ALONE_MIN_ELEMENTS if out is None else 1):
+    wider than the library's grid are torch's as well, and few elements without a rectifier, unless
+    the pass is captured into a graph."""
+    n = grad.numel()
+    if n == 0 or not grad.is_cuda:
+        return False
+    # (a captured pass has no host to spare work for, and torch's sum would leave a memset in the graph)
+    if out is None and n < _BIAS_ALONE_MIN_ELEMENTS and not torch.cuda.is_current_stream_capturing():
         return False
     if torch.is_grad_enabled() or torch._C._len_torch_dispatch_stack():
         return False
@@ -183,8 +188,9 @@ def _epilogue_backward(grad, out, bias, act):
                                               functors.ACTIVATIONS[act])
     if act == "relu":
         grad = grad * (out > 0)
-    grad_bias = grad.reshape(-1, grad.shape[-1]).sum(0) if bias is not None else None
-    return grad, grad_bias
+    if bias is None:
+        return grad, None
+    return grad, (grad if grad.dim() == 2 else grad.reshape(-1, grad.shape[-1])).sum(0)
 
 
 class _ConvamBiasAct(torch.autograd.Function):

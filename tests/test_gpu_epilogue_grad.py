@@ -57,3 +57,21 @@ def test_small_gradients_of_a_bias_alone_stay_with_torch(monkeypatch, rows, cols
     assert torch.equal(z, want) and len(seen) == calls
     # (any order of the sum: n * 2^-24 * sum|terms|)
     assert ((b.double() - want.double().sum(0)).abs() <= rows * 2.0 ** -24 * want.double().abs().sum(0)).all()
+
+
+def test_captured_bias_gradient_replays():
+    """A captured pass stays with the library at every size: torch's sum over many blocks clears its
+    counters by a recorded memset."""
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    grad = torch.randn((2048, 256), device="cuda", generator=gen)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        captured = layers._epilogue_backward(grad, None, True, None)[1]
+    for i in range(4):
+        grad.copy_(torch.randn((2048, 256), device="cuda", generator=gen))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, functors.epilogue_grad(grad, None, True, None)[1]), i
+        (grad * 2).sum(0)  # (eager work between the replays)
+        torch.cuda.synchronize()
