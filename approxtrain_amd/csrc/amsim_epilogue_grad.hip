@@ -6,15 +6,15 @@
 // rows of up to 64 columns; its threads run along the columns first, 16 lanes or more, and each adds every
 // (256 / columns)-th row in four chains.  Rows of fewer than 16 columns leave lanes idle (6 columns: ten of
 // 16) and are read in short pieces, which a narrow output's few bytes bear.  The slabs' sums go to the workspace and
-// the fixed-order reduction adds them (one slab writes the bias gradient itself): no atomics, no counter to
-// clear, the same bits on every run.
-// On the device, torch's compare, product with the mask and sum against this file: 25600 x 16 18.4 -> 8.4 us,
-// 401408 x 6 30.6 -> 13.6, 8192 x 512 37.7 -> 14.7 (3.4 TB/s), 401408 x 128 257 -> 129 (4.8 TB/s); the sum alone
-// 8192 x 512 17.8 -> 8.1, 401408 x 128 52.4 -> 37.3 (5.5 TB/s).  Training step of the 32 x 256 x 512 attention block
+// slab_sum_kernel adds them (one slab writes the bias gradient itself): no atomics, no counter to clear, the
+// same bits on every run.  Chains run in 32 bits, what combines them in 64: added in 32 bits, a narrow output's
+// 32 ways were the largest error (25600 x 16, terms of mean 0.3: 7.9e-8 of the result; 1.8e-8 now, torch's sum 2.9e-8).
+// On the device, torch's compare, product with the mask and sum against this file: 25600 x 16 18.3 -> 7.5 us,
+// 401408 x 6 30.4 -> 13.5, 8192 x 512 37.7 -> 13.7 (3.7 TB/s), 401408 x 128 257 -> 130 (4.7 TB/s); the sum alone
+// 8192 x 512 18.2 -> 7.0, 401408 x 128 52.6 -> 37.7 (5.5 TB/s).  Training step of the 32 x 256 x 512 attention block
 // (four biases) 2711 -> 2661 us; LeNet-5's convolutions, bound by the host, show no difference beyond their spread.
 #include "amsim_internal.h"
 #include "amsim_device.h"
-#include "amsim_gemm_common.h"
 
 #include <algorithm>
 
@@ -49,7 +49,7 @@ template <int TX, bool RELU>
 __global__ __launch_bounds__(WG) void epilogue_grad_kernel(EpilogueGradArgs a)
 {
     constexpr int TY = WG / TX;
-    __shared__ float part[TY][TX];
+    __shared__ double part[TY][TX];
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
     const int64_t col = (int64_t)blockIdx.x * TX + tx;
     const int64_t beg = (int64_t)blockIdx.y * a.rows_per_slab;
@@ -73,13 +73,43 @@ __global__ __launch_bounds__(WG) void epilogue_grad_kernel(EpilogueGradArgs a)
         }
     }
     if (a.partial == nullptr) return;  // (the same for every thread)
-    part[ty][tx] = (c[0] + c[1]) + (c[2] + c[3]);
+    part[ty][tx] = ((double)c[0] + c[1]) + ((double)c[2] + c[3]);
     __syncthreads();
     if (ty == 0 && col < a.cols) {
-        float s = part[0][tx];
+        double s = part[0][tx];
 #pragma unroll
         for (int w = 1; w < TY; ++w) s += part[w][tx];
-        a.partial[(int64_t)blockIdx.y * a.cols + col] = s;
+        a.partial[(int64_t)blockIdx.y * a.cols + col] = (float)s;
+    }
+}
+
+// OUTS columns per workgroup, WG / OUTS threads ("ways") per column, eight loads of each in flight: few columns
+// with many slabs use OUTS = 8, else the loop over the slabs is one long chain of memory latencies.
+template <int OUTS>
+__global__ __launch_bounds__(WG) void slab_sum_kernel(const float *partial, float *grad_bias, int slabs, int cols)
+{
+    constexpr int WAYS = WG / OUTS;
+    __shared__ double part[WAYS][OUTS];
+    const int o = threadIdx.x % OUTS, way = threadIdx.x / OUTS;
+    const int64_t col = (int64_t)blockIdx.x * OUTS + o;
+    double c[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (col < cols) {
+        const float *src = partial + col;
+        for (int sl = way; sl < slabs; sl += 8 * WAYS) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)min(sl + u * WAYS, slabs - 1) * cols];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) c[u] += sl + u * WAYS < slabs ? v[u] : 0.0f;  // (no load waits for a test)
+        }
+    }
+    part[way][o] = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+    __syncthreads();
+    if (way == 0 && col < cols) {
+        double s = part[0][o];
+#pragma unroll
+        for (int w = 1; w < WAYS; ++w) s += part[w][o];
+        grad_bias[col] = (float)s;
     }
 }
 
@@ -132,14 +162,10 @@ int amsim_epilogue_grad_f32(const float *grad, const float *out, int64_t rows, i
     }
     AMSIM_HIP_CHECK(hipGetLastError());
     if (!grad_bias || slabs == 1) return AMSIM_OK;
-    RArgs ra{};
-    ra.partial = a.partial;
-    ra.out = grad_bias;
-    ra.R = 1; ra.J = cols; ra.Rp = 1; ra.Jp = cols;
-    ra.so_r = cols; ra.so_j = 1;
-    ra.nsplit = (int)slabs;
-    ra.batch = 1;
-    launch_reduce(ra, s);
+    if (cols <= 16384 && slabs >= 64)
+        slab_sum_kernel<8><<<(unsigned)((cols + 7) / 8), WG, 0, s>>>(partial, grad_bias, (int)slabs, cols);
+    else
+        slab_sum_kernel<64><<<(unsigned)((cols + 63) / 64), WG, 0, s>>>(partial, grad_bias, (int)slabs, cols);
     AMSIM_HIP_CHECK(hipGetLastError());
     return AMSIM_OK;
 }

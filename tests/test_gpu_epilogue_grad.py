@@ -75,3 +75,14 @@ def test_captured_bias_gradient_replays():
         assert torch.equal(captured, functors.epilogue_grad(grad, None, True, None)[1]), i
         (grad * 2).sum(0)  # (eager work between the replays)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows,cols", [(25600, 16), (200704, 6), (401408, 16), (262144, 100), (50000, 600)])
+def test_error_against_64_bits(rows, cols):
+    """Positive terms, 100 slabs of rows and more: a slab's rounding errors average out over the slabs, so what is
+    left is the one rounding of the result, at most 2^-24 of each column's sum."""
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    grad = torch.rand((rows, cols), device="cuda", generator=gen)
+    want = grad.double().sum(0)
+    got = functors.epilogue_grad(grad, None, True, None)[1].double()
+    assert (got - want).norm() <= 2.0 ** -24 * want.norm()
