@@ -4,6 +4,7 @@ argument meaning, operating on CUDA/HIP torch tensors.  torch supplies device
 memory, the workspace and the current stream; all arithmetic happens in
 libamsim.so."""
 import ctypes as C
+import functools
 
 import torch
 
@@ -332,6 +333,11 @@ def epilogue_grad(grad, out, has_bias, activation):
     return epilogue_grad_checked(grad, out, has_bias, act)
 
 
+@functools.lru_cache(maxsize=256)
+def _epilogue_grad_workspace(rows, cols):
+    return load_library().amsim_epilogue_grad_workspace_bytes(rows, cols)
+
+
 def epilogue_grad_checked(grad, out, has_bias, act):
     """The same for operands known to be what the library takes: contiguous 32-bit floats in the memory
     of one device, of one shape and not empty; ``act`` is the activation's code.  (A small training step
@@ -341,7 +347,7 @@ def epilogue_grad_checked(grad, out, has_bias, act):
     grad_z = torch.empty_like(grad) if act else grad
     grad_bias = grad.new_empty(cols) if has_bias else None
     lib = load_library()
-    nbytes = lib.amsim_epilogue_grad_workspace_bytes(rows, cols) if has_bias else 0
+    nbytes = _epilogue_grad_workspace(rows, cols) if has_bias else 0
     # (torch's allocations start on 512-byte boundaries)
     ws = grad.new_empty(nbytes // 4) if nbytes else None
     check(lib.amsim_epilogue_grad_f32(grad.data_ptr(), out.data_ptr() if act else None, rows, cols, act,

@@ -148,13 +148,16 @@ def _plain_memory(t):
         return False
 
 
-# A bias alone is one sum over the rows, a single call of torch: 6.4 to 10 us of host work against the
-# library's 10.9 (two launches, two allocations), which the small steps, bound by the host, cannot hide.
-# Back to back, torch / library: 128 x 1024 6.7 / 11.2 us, 1024 x 1024 10.3 / 11.3, 1024 x 2048 11.3 / 11.3,
-# 512 x 4096 10.7 / 11.1, 4096 x 512 16.8 / 11.3, 401408 x 16 13.0 / 11.1, 8192 x 512 16.8 / 11.2; on the device alone the
-# library is ahead from 2^17 elements on.  With the rectifier torch takes three calls, 15.4 us on the
-# host from 1 x 1 on against 8.4 (one slab of rows) and 12.
-_BIAS_ALONE_MIN_ELEMENTS = 1 << 21
+# A bias alone is one sum over the rows, a single call of torch: 5.6 to 8.8 us of host work against the
+# library's 10.2 (two launches, two allocations), which the small steps, bound by the host, cannot hide.
+# Back to back, torch / library: 128 x 1024 6.2 / 10.3 us, 4096 x 64 9.1 / 10.6, 256 x 4096 8.8 / 10.5,
+# 1024 x 1024 9.9 / 10.5, 2048 x 512 11.5 / 10.4, 4096 x 256 14.8 / 10.6, 8192 x 512 16.8 / 10.5.  On the device
+# alone the library is ahead from 2^17 elements on (1024 x 512: 10.2 / 5.9), which counts once the products
+# beside it take longer than the host does: attention's training step over 8 x 128 positions of depth 512
+# (2^19 elements) 660 us with torch's sum and 644 with the library's in processes whose host is fast,
+# 32 x 128 of depth 128 704 and 709 where it is slow.  With the rectifier torch takes three calls, 15 us on the
+# host from 1 x 1 on against 8.4 (one slab of rows) and 11.5.
+_BIAS_ALONE_MIN_ELEMENTS, _BIAS_ALONE_MIN_ROWS = 1 << 19, 1024
 
 
 def _library_epilogue(grad, out):
@@ -168,8 +171,9 @@ def _library_epilogue(grad, out):
     if n == 0 or not grad.is_cuda:
         return False
     # (a captured pass has no host to spare work for, and torch's sum would leave a memset in the graph)
-    if out is None and n < _BIAS_ALONE_MIN_ELEMENTS and not torch.cuda.is_current_stream_capturing():
-        return False
+    if out is None and (n < _BIAS_ALONE_MIN_ELEMENTS or n < _BIAS_ALONE_MIN_ROWS * grad.shape[-1]):
+        if not torch.cuda.is_current_stream_capturing():
+            return False
     if torch.is_grad_enabled() or torch._C._len_torch_dispatch_stack():
         return False
     if not _plain_memory(grad) or grad.shape[-1] >= 1 << 30 or forward_ad.unpack_dual(grad).tangent is not None:
